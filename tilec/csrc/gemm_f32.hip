@@ -514,6 +514,35 @@ hipError_t launch_gemm_f32_pad(const MatmulArgs& a) {
   }
 }
 
+template <int BM, int BN, int BK, int WM, int WN, int PF, int WPE, bool LOW>
+hipError_t launch_gemm_f32_x6(const MatmulArgs& a);  // gemm_f32_x6.hip
+template <int W>
+hipError_t launch_gemm_f32_x6_direct(const MatmulArgs& a);
+
+namespace {
+
+// Byte offsets within a K step of gemm_f32_x6.hip take 31 bits ((rows of the
+// tile along the stride) * ld * 4); beyond that the register-staged kernel of
+// the same tile, K step and waves (so a K split is the same in both).
+template <int BM, int BN, int BK, int WM, int WN, int PF, int WPE, bool LOW>
+hipError_t launch_gemm_f32_planes(const MatmulArgs& a) {
+  constexpr int64_t lim = (int64_t(1) << 31) - 4096;
+  const int64_t r1 = (a.layout & TILEC_X1_COL_MAJOR) ? BK : BM, r2 = (a.layout & TILEC_X2_COL_MAJOR) ? BN : BK;
+  if (r1 * a.ldx1 * 4 >= lim || r2 * a.ldx2 * 4 >= lim) return launch_gemm_f32<BM, BN, BK, WM, WN>(a);
+  return launch_gemm_f32_x6<BM, BN, BK, WM, WN, PF, WPE, LOW>(a);
+}
+
+// The same for the kernel whose waves share K (64 x 64 tiles, K step 16).
+template <int W>
+hipError_t launch_gemm_f32_planes_direct(const MatmulArgs& a) {
+  constexpr int64_t lim = (int64_t(1) << 31) - 4096;
+  const int64_t r1 = (a.layout & TILEC_X1_COL_MAJOR) ? 16 : 64, r2 = (a.layout & TILEC_X2_COL_MAJOR) ? 64 : 16;
+  if (r1 * a.ldx1 * 4 >= lim || r2 * a.ldx2 * 4 >= lim) return launch_gemm_f32_unsplit(a);
+  return launch_gemm_f32_x6_direct<W>(a);
+}
+
+}  // namespace
+
 // Variant table for this family (its order is part of the variant numbering).
 const VariantDesc* gemm_f32_variants(int* count) {
   static const VariantDesc t[] = {
@@ -555,6 +584,24 @@ const VariantDesc* gemm_f32_variants(int* count) {
        launch_gemm_f32_pad<128, 128, 32, 3, 2, 4>, 0, pad_workspace_bytes, pad_counter_bytes},
       {"gemm_f32_64x64x32_w2x2_pad", TILEC_FAMILY_GEMM, TILEC_F32, 64, 64, 32, 4, 0, 3,
        launch_gemm_f32_pad<64, 64, 32, 3, 2, 2>, 0, pad_workspace_bytes, pad_counter_bytes},
+  };
+  *count = (int)(sizeof(t) / sizeof(t[0]));
+  return t;
+}
+
+// The plane variants (three bf16 planes a value on the bf16 MFMAs,
+// gemm_f32_x6.hip), a table of their own behind the others: variant numbers
+// in use stay what they are.  `unroll` is the number of LDS stages.
+const VariantDesc* gemm_f32_x6_variants(int* count) {
+  static const VariantDesc t[] = {
+      {"gemm_f32_256x256x16_x6", TILEC_FAMILY_GEMM, TILEC_F32, 256, 256, 16, 8, 0, 3,
+       launch_gemm_f32_planes<256, 256, 16, 2, 4, 1, 1, false>},
+      {"gemm_f32_128x128x16_x6", TILEC_FAMILY_GEMM, TILEC_F32, 128, 128, 16, 4, 0, 3,
+       launch_gemm_f32_planes<128, 128, 16, 2, 2, 1, 2, true>},
+      {"gemm_f32_128x128x32_w8_x6", TILEC_FAMILY_GEMM, TILEC_F32, 128, 128, 32, 8, 0, 3,
+       launch_gemm_f32_planes<128, 128, 32, 2, 4, 4, 1, true>},
+      {"gemm_f32_64x64x16_d4_x6", TILEC_FAMILY_GEMM, TILEC_F32, 64, 64, 16, 4, 0, 2,
+       launch_gemm_f32_planes_direct<4>},
   };
   *count = (int)(sizeof(t) / sizeof(t[0]));
   return t;

@@ -107,6 +107,8 @@ def hip_configs(M, K, N, dtype="f32", layout=None):
             continue  # the panel kernel reads a row-major x2 (it runs the streaming kernel otherwise)
         if pad_variant(v) and not needs_pad(M, K, N, layout, code):
             continue  # aligned operands: the direct-to-LDS variants read them in place
+        if planes_variant(v) and M <= 16:
+            continue  # bound by reading x2: the streaming and direct kernels' work
         if v["family"] == _lib.FAMILY_SKINNY and rows_variant(v):
             epl = 4 if code == _lib.F32 else 8  # elements per 16-byte load
             row_tile = v["name"].endswith(("_c128", "_c256"))  # the row-dot kernel takes any K
@@ -189,6 +191,12 @@ def pad_variant(v):
     direct-to-LDS tile kernel (csrc/gemm_f32.hip, launch_gemm_f32_pad;
     csrc/gemm_bf16.hip, launch_gemm_bf16_pad)."""
     return v["name"].endswith("_pad")
+
+
+def planes_variant(v):
+    """Variants named *_x6 split fp32 values into three bf16 planes and run the
+    six plane products on the bf16 MFMAs (csrc/gemm_f32_x6.hip)."""
+    return v["name"].endswith("_x6")
 
 
 def needs_pad(M, K, N, layout=None, dtype="f32"):

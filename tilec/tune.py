@@ -96,7 +96,8 @@ def roofline(M, K, N, cus, dtype, kernel, split_k, layout=0):
     tail = wgs / (rounds * slots)
     fill = min(1.0, wgs / cus)
     pad = (M * N) / max(1, tiles * bm * bn)
-    t_c = 2.0 * M * N * K / (PEAK_FLOPS[dtype] * max(fill * pad, 1e-9))
+    peak = PEAK_FLOPS["bf16"] / 6 if kernel.endswith("_x6") else PEAK_FLOPS[dtype]  # six plane products
+    t_c = 2.0 * M * N * K / (peak * max(fill * pad, 1e-9))
     t_m = (esz * (M * K + K * N) + 4 * M * N + (8.0 * tiles * bm * bn * split_k if split_k > 1 else 0)) / PEAK_HBM
     t_r = esz * (M * K * cdiv(N, bn) + K * N * cdiv(M, bm)) / PEAK_L2_READ
     launches, moved = prepass(M, K, N, dtype, kernel, layout)
@@ -118,8 +119,9 @@ def features(M, K, N, cus, dtype, kernel, split_k, layout=0):
     row-tile kernels take only such operands and run a slower fallback of
     the same tile for the others, a difference the sizes alone do not show
     the trees (on MI355X it took the held-out worst case from 2.3x to 1.5x).
-    Then three variant properties the descriptor sizes do not carry: 16x16
-    MFMA blocks (`*_m16`), operands transposed (`*_kc`) or padded (`*_pad`)
+    Then three variant properties the descriptor sizes do not carry: another
+    MFMA form than the type's plain tiles (16x16 blocks, `*_m16`, for bf16;
+    bf16 planes, `*_x6`, for fp32), operands transposed (`*_kc`) or padded (`*_pad`)
     into the workspace first — otherwise such a variant and its plain
     counterpart look the same to the trees.  Last, whether this config runs
     a slower fallback of its tile for these operands (`falls_back`): the
@@ -141,7 +143,7 @@ def features(M, K, N, cus, dtype, kernel, split_k, layout=0):
             ls(t_est), ls(t_c), ls(t_m), ls(t_r), pad, tail, fill, lg(kpw), rounds,
             float(aligned(M if layout & _lib.X1_COL_MAJOR else K, dtype)),
             float(aligned(K if layout & _lib.X2_COL_MAJOR else N, dtype)),
-            float("_m16" in kernel), float(kernel.endswith("_kc")), float(kernel.endswith("_pad")),
+            float("_m16" in kernel or kernel.endswith("_x6")), float(kernel.endswith("_kc")), float(kernel.endswith("_pad")),
             float(falls_back(kernel, M, K, N, dtype, layout))]
 
 
@@ -383,7 +385,22 @@ def _bf16_stream(rng, count):
     return got
 
 
-def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_narrow=60, n_bf16=80):
+def _mixed_stream(rng, count, dtype):
+    """Products of one dtype in every layout: M in [17, 4096], K and N in
+    [64, 8192] log-uniform, half of the K and N multiples of 64 as layer
+    widths are — linear layers' forward and gradient products, where tile,
+    plane, split and alignment choices all meet."""
+    size = lambda lo, hi: round(2 ** rng.uniform(math.log2(lo), math.log2(hi)))
+    width = lambda v: v // 64 * 64 if v > 64 and rng.random() < 0.5 else v
+    got = set()
+    while len(got) < count:
+        M, K, N = size(17, 4096), width(size(64, 8192)), width(size(64, 8192))
+        if 1 << 20 <= M * K * N <= 1 << 34 and max(M * K, K * N, M * N) <= 1 << 25:
+            got.add((M, K, N, dtype, rng.choice((0, 1, 2, 2, 3))))
+    return got
+
+
+def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_narrow=60, n_bf16=80, n_mixed=0):
     """Seeded random shapes (M, K, N, dtype, layout): `n` row-major draws plus
     CONFIG_SHAPES, `n_layout` draws of a second stream (seed + 1) with a
     random non-row-major layout, plus LAYOUT_CONFIG_SHAPES, `n_rows` x @ W.T
@@ -391,7 +408,8 @@ def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_nar
     domain, `n_tile` x @ W.T shapes with 5 <= M <= 16 from a fourth
     (seed + 3), the row-tile kernel's, row-major `n_medium` medium
     outputs (seed + 4) and `n_narrow` narrow outputs over a long K
-    (seed + 5), and `n_bf16` bf16 tile GEMMs in random layouts (seed + 6).
+    (seed + 5), `n_bf16` bf16 tile GEMMs in random layouts (seed + 6), and
+    `n_mixed` products of each dtype in random layouts (seed + 7, + 8).
     None of UNSEEN_SHAPES is ever included."""
     rng = random.Random(seed)
     out = set(CONFIG_SHAPES)
@@ -422,6 +440,7 @@ def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_nar
     more = {t + (0,) for t in _medium_stream(random.Random(seed + 4), n_medium) |
             _narrow_stream(random.Random(seed + 5), n_narrow)}
     more |= _bf16_stream(random.Random(seed + 6), n_bf16)
+    more |= _mixed_stream(random.Random(seed + 7), n_mixed, "f32") | _mixed_stream(random.Random(seed + 8), n_mixed, "bf16")
     unseen = {u + (0,) for u in UNSEEN_SHAPES}
     return sorted((out | lay | rows | tile | more) - unseen, key=lambda s: (s[0] * s[1] * s[2], s))
 
@@ -469,7 +488,7 @@ def bench(n=300, seed=0, path=None):
         if not rows:
             w.writerow(FIELDS)
         g = torch.Generator(device="cuda").manual_seed(seed)
-        todo = shapes(n, seed)
+        todo = shapes(n, seed, n_mixed=200)
         for i, (M, K, N, dtype, layout) in enumerate(todo):
             have = timed_cfgs.get((M, K, N, dtype, layout), {})
             missing = [c for c in ext.hip_configs(M, K, N, dtype, layout) if c not in have]
@@ -554,6 +573,45 @@ def _key(r):
     return (int(r["M"]), int(r["K"]), int(r["N"]), r["dtype"], int(r["layout"]))
 
 
+KEEP_WITHIN, KEEP_WORST = 1.002, 1.08  # candidates(): geometric mean and worst case over one dtype's shapes
+
+
+def candidates(rows):
+    """Names of the variants `pick` chooses among: every variant of a dtype
+    whose removal would cost more than the others can make up.  Starting from
+    all of them, the variant whose loss raises the geometric mean (over the
+    timed shapes) of best-with-the-rest over best the least is dropped, until
+    that mean would pass KEEP_WITHIN or a shape KEEP_WORST.  Near-copies of a variant win a shape by
+    less than timings repeat, and each one more is one more way for a
+    prediction to be too low."""
+    keep = set()
+    for dtype in sorted({r["dtype"] for r in rows}):
+        times = {}  # shape -> variant -> its best ms
+        for r in rows:
+            if r["dtype"] == dtype:
+                t = times.setdefault(_key(r), {})
+                t[r["kernel"]] = min(t.get(r["kernel"], math.inf), r["ms"])
+        left = {k for t in times.values() for k in t}
+        floor = {k: min(t.values()) for k, t in times.items()}
+
+        def cost(names):
+            total = 0.0
+            for k, t in times.items():
+                ms = [v for n, v in t.items() if n in names]
+                if not ms or min(ms) > KEEP_WORST * floor[k]:
+                    return math.inf
+                total += math.log(min(ms) / floor[k])
+            return math.exp(total / len(times))
+
+        while len(left) > 1:
+            c, drop = min((cost(left - {n}), n) for n in left)
+            if c > KEEP_WITHIN:
+                break
+            left.remove(drop)
+        keep |= left
+    return keep
+
+
 def train(test_frac=0.2, seeds=(0, 1, 2), out=MODEL, path=None):
     """Fit on log(ms); report held-out quality against the best config and the
     library's built-in rule over several random 80/20 splits of the shapes
@@ -567,14 +625,19 @@ def train(test_frac=0.2, seeds=(0, 1, 2), out=MODEL, path=None):
     rows = [r for r in rows if r["kernel"] in names and
             (not ext.rows_variant(names[r["kernel"]]) or
              (r["kernel"], int(r["split_k"])) in ext.hip_configs(*_key(r)[:4], int(r["layout"])))]
+    keep = candidates(rows)
+    print(f"{len(keep)} of {len({r['kernel'] for r in rows})} variants kept: {sorted(keep)}", flush=True)
+    all_rows, rows = rows, [r for r in rows if r["kernel"] in keep]
     feats = {id(r): row_features(r) for r in rows}
 
     def data(rs):
         return [feats[id(r)] for r in rs], [math.log(max(r["ms"], 1e-6)) for r in rs]
 
-    by_shape = {}
+    by_shape, best_ms = {}, {}
     for r in rows:
         by_shape.setdefault(_key(r), []).append(r)
+    for r in all_rows:  # the best of every variant, kept or not
+        best_ms[_key(r)] = min(best_ms.get(_key(r), math.inf), r["ms"])
     tests = []
     for seed in seeds:
         keys = sorted(by_shape)
@@ -587,20 +650,23 @@ def train(test_frac=0.2, seeds=(0, 1, 2), out=MODEL, path=None):
     with multiprocessing.get_context("fork").Pool(min(len(jobs), os.cpu_count() or 1)) as pool:
         models = pool.map(_fit_gbr, jobs)
     L = _lib.lib()
+    auto_rows = {}
+    for r in all_rows:
+        auto_rows.setdefault(_key(r), []).append(r)
     gm = lambda v: math.exp(sum(math.log(a) for a in v) / len(v)) if v else float("nan")
     splits = []
     for seed, test, model in zip(seeds, tests, models):
         ratio_model, ratio_default, worst = [], [], None
         for k in sorted(test):
             rs = by_shape[k]
-            best = min(r["ms"] for r in rs)
+            best = best_ms[k]
             pred = model.predict([feats[id(r)] for r in rs])
             chosen = rs[min(range(len(rs)), key=lambda i: pred[i])]
             M, K, N, dtype, layout = k
             dcode = _lib.F32 if dtype == "f32" else _lib.BF16
             auto = _lib.variants()[L.tilec_select_variant_layout(M, N, K, dcode, layout, 0, 0)]["name"]
             auto_split = L.tilec_auto_split_k(M, N, K, dcode, _lib.variant_id(auto))
-            default = [r for r in rs if r["kernel"] == auto and int(r["split_k"]) == auto_split]
+            default = [r for r in auto_rows.get(k, ()) if r["kernel"] == auto and int(r["split_k"]) == auto_split]
             ratio_model.append(chosen["ms"] / best)
             if worst is None or ratio_model[-1] > worst[0]:
                 worst = (ratio_model[-1], list(k), [chosen["kernel"], int(chosen["split_k"])])
@@ -625,7 +691,7 @@ def train(test_frac=0.2, seeds=(0, 1, 2), out=MODEL, path=None):
     print(f"over {len(splits)} splits: model {report['model_geomean_vs_best']:.3f}x (geo mean of geo means), "
           f"worst {report['model_worst_vs_best']:.2f}x; builtin {report['builtin_geomean_vs_best']:.3f}x, "
           f"worst {report['builtin_worst_vs_best']:.2f}x")
-    export(models[-1], out, report, best_table(rows))
+    export(models[-1], out, report, best_table(all_rows), sorted(keep))
     return report
 
 
@@ -636,7 +702,7 @@ def _fit_gbr(job):
     with depth 4; depth 8 overfits (worst 10x)."""
     from sklearn.ensemble import GradientBoostingRegressor
     X, y, seed = job
-    return GradientBoostingRegressor(n_estimators=300, max_depth=6, learning_rate=0.05, random_state=seed).fit(X, y)
+    return GradientBoostingRegressor(n_estimators=500, max_depth=6, learning_rate=0.05, random_state=seed).fit(X, y)
 
 
 def best_table(rows):
@@ -649,9 +715,10 @@ def best_table(rows):
     return {",".join(map(str, k)): [r["kernel"], int(r["split_k"])] for k, r in sorted(best.items())}
 
 
-def export(model, path, report=None, table=None):
+def export(model, path, report=None, table=None, keep=None):
     """Write a fitted GradientBoostingRegressor as plain JSON trees, plus the
-    measured best config of every benchmarked shape (`table`)."""
+    measured best config of every benchmarked shape (`table`) and the variants
+    to choose among (`keep`; None: all)."""
     trees = []
     for est in model.estimators_[:, 0]:
         t = est.tree_
@@ -664,7 +731,7 @@ def export(model, path, report=None, table=None):
         model._raw_predict_init([[0.0] * model.n_features_in_])[0][0])
     data = {"format": "gbr-trees-v1", "learning_rate": model.learning_rate, "init": init,
             "n_features": int(model.n_features_in_), "trees": trees, "report": report or {},
-            "best": table or {}}
+            "best": table or {}, "keep": keep}
     with open(path, "w") as f:
         json.dump(data, f)
 
@@ -679,6 +746,7 @@ class TreeModel:
         self.n_features = data["n_features"]
         self.trees = [{k: np.asarray(t[k]) for k in ("left", "right", "feature", "threshold", "value")}
                       for t in data["trees"]]
+        self.keep = frozenset(data["keep"]) if data.get("keep") else None
         self.report = data.get("report", {})  # held-out quality at training time
         self.best = {}
         for k, v in data.get("best", {}).items():
@@ -728,6 +796,8 @@ def pick(M, K, N, dtype="f32", layout=0):
     measured = model.best.get((M, K, N, dtype, layout))
     if measured is not None and measured in cands:
         return measured
+    if model.keep is not None:
+        cands = [c for c in cands if c[0] in model.keep] or cands
     cus = _cus()
     if model.n_features < len(features(M, K, N, cus, dtype, cands[0][0], cands[0][1], layout)):
         return None  # a model trained on fewer features than these: use the built-in rule
