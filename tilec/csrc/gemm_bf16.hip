@@ -232,13 +232,46 @@ hipError_t launch_one(const MatmulArgs& a, dim3 grid) {
 
 template <int BM, int BN, int BK, int NBUF, int WM, int WN, bool CA, bool CB, int MF>
 hipError_t launch_gemm_bf16_lds(const MatmulArgs& a);  // gemm_bf16_lds.hip
+template <int BM, int BN, int WM, int WN, int PF, int WPE>
+hipError_t launch_gemm_bf16_any(const MatmulArgs& a);  // gemm_bf16_any.hip
 
 namespace {
 
+// Whether the kernel of gemm_bf16_any.hip (tiles of up to 128 rows) takes
+// these operands: its straddling loads need 8 elements along K and two along
+// an r-contiguous extent, its offsets within a K step 31 bits.
+bool any_takes(const MatmulArgs& a) {
+  constexpr int64_t lim = (int64_t(1) << 31) - 4096;
+  const bool ca = a.layout & TILEC_X1_COL_MAJOR, cb = a.layout & TILEC_X2_COL_MAJOR;
+  return a.K >= 8 && (!ca || a.M >= 2) && (cb || a.N >= 2) && 128 * a.ldx1 * 2 < lim && 128 * a.ldx2 * 2 < lim;
+}
+
+// Unaligned operands of a variant whose own kernel needs aligned ones, K not
+// split: tiles of 128 x 128 where they give every CU one, else 64 x 64 (the
+// generic kernel's 128 x 128 tile of 2-byte loads, on MI355X: 2048 x 1024 x
+// 1024 with an x1 row stride of 1025, 43 against 17 us; 300 x 512 x 1024 with
+// one of 513, 44 against 6.8; 4096 x 1024 x 4096 with one of 1027, 174 against
+// 80).  A split keeps the variant's own tile, which its workspace is sized for.
+template <int BM, int BN, int WM, int WN>
+bool launch_unaligned(const MatmulArgs& a, hipError_t& e) {
+  if (!any_takes(a)) return false;
+  if (gemm_split_geom(a.K, 64, a.split_k).splits <= 1) {
+    e = cdiv(a.M, 128) * cdiv(a.N, 128) >= 256 ? launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a)
+                                               : launch_gemm_bf16_any<64, 64, 2, 2, 4, 2>(a);
+    return true;
+  }
+  if constexpr (BM == 128 && BN == 128 && WM == 2 && WN == 4) e = launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a);
+  else if constexpr (BM == 128 && BN == 64 && WM == 2 && WN == 2) e = launch_gemm_bf16_any<128, 64, 2, 2, 2, 2>(a);
+  else if constexpr (BM == 64 && BN == 64 && WM == 2 && WN == 2) e = launch_gemm_bf16_any<64, 64, 2, 2, 4, 2>(a);
+  else return false;
+  return true;
+}
+
 // Aligned operands (16-byte base, K, N, lda, ldb multiples of 8) whose tile
 // offsets fit 32 bits run the LDS-DMA kernel of gemm_bf16_lds.hip with a
-// ring of NBUF stage buffers of BK; everything else runs the generic kernel
-// above with the same output tile (NBUF == 0: generic kernel only).  Both
+// ring of NBUF stage buffers of BK; unaligned ones that of gemm_bf16_any.hip;
+// what neither takes runs the generic kernel above with the same output tile
+// (aligned operands too where NBUF == 0).  Both
 // use the variant's WM x WN waves, so a K split is possible in one exactly
 // when it is in the other.
 template <int BM, int BN, int BK, int NBUF, int WM, int WN, bool CA, bool CB, int MF>
@@ -259,6 +292,10 @@ hipError_t launch_layout(const MatmulArgs& a) {
     if (vec && a_rows * a.ldx1 * 2 < (int64_t(1) << 31) - 4096 && b_rows * a.ldx2 * 2 < (int64_t(1) << 31) - 4096)
       return launch_gemm_bf16_lds<BM, BN, BK, NBUF, WM, WN, CA, CB, MF>(a);
   }
+  if (!vec) {
+    hipError_t e = hipSuccess;
+    if (launch_unaligned<BM, BN, WM, WN>(a, e)) return e;
+  }
   dim3 grid((unsigned)tiles);
   return vec ? launch_one<BM, BN, 64, WM, WN, true, CA, CB>(a, grid)
              : launch_one<BM, BN, 64, WM, WN, false, CA, CB>(a, grid);
@@ -266,9 +303,9 @@ hipError_t launch_layout(const MatmulArgs& a) {
 
 // Aligned operands (16-byte base, contiguous extents and strides multiples
 // of 8) whose tile offsets fit 32 bits run the LDS-DMA kernel of
-// gemm_bf16_lds.hip with a ring of NBUF stage buffers of BK; everything else
-// runs the generic kernel above with the same output tile (NBUF == 0: generic
-// kernel only).  Both use the variant's WM x WN waves, so a K split is
+// gemm_bf16_lds.hip with a ring of NBUF stage buffers of BK; unaligned ones
+// that of gemm_bf16_any.hip; what neither takes runs the generic kernel above
+// with the same output tile (aligned operands too where NBUF == 0).  All use the variant's WM x WN waves, so a K split is
 // possible in one exactly when it is in the other.
 template <int BM, int BN, int BK, int NBUF, int WM = 2, int WN = 2, int MF = 32>
 hipError_t launch_gemm_bf16(const MatmulArgs& a) {
@@ -503,4 +540,45 @@ const VariantDesc* gemm_bf16_variants(int* count) {
   *count = (int)(sizeof(t) / sizeof(t[0]));
   return t;
 }
+
+namespace {
+
+template <int BM, int BN, int WM, int WN, int PF, int WPE>
+hipError_t launch_any_or_generic(const MatmulArgs& a) {
+  return any_takes(a) ? launch_gemm_bf16_any<BM, BN, WM, WN, PF, WPE>(a) : launch_gemm_bf16<BM, BN, 64, 0, WM, WN>(a);
+}
+
+}  // namespace
+
+// Tiles of 64 and 128 on four waves, two or more workgroups a CU, for outputs
+// that 256- and 8-wave 128-tiles cut into too few pieces: those then split K
+// 8 or 16 ways, and the last workgroup of each tile reads the other splits'
+// partial tiles alone (448 KiB at 128 x 4096 x 4096, 8 splits of 128 x 128)
+// while the other CUs are idle.  On MI355X, 128 x 4096 x 4096 (x2
+// column-major): 18.9 us so, 12.0 in 64 x 64 tiles with two splits; 1024^3,
+// 64 against 256 workgroups: 9.7 and 6.7 us.  A table of its own behind the
+// others (variant numbers in use stay what they are).
+const VariantDesc* gemm_bf16_small_variants(int* count) {
+  static const VariantDesc t[] = {
+      {"gemm_bf16_64x64x64_r4_m16", TILEC_FAMILY_GEMM, TILEC_BF16, 64, 64, 64, 4, 0, 4,
+       launch_gemm_bf16<64, 64, 64, 4, 2, 2, 16>},
+      {"gemm_bf16_128x64x64_r3_m16", TILEC_FAMILY_GEMM, TILEC_BF16, 128, 64, 64, 4, 0, 3,
+       launch_gemm_bf16<128, 64, 64, 3, 2, 2, 16>},
+      {"gemm_bf16_64x128x64_r3_m16", TILEC_FAMILY_GEMM, TILEC_BF16, 64, 128, 64, 4, 0, 3,
+       launch_gemm_bf16<64, 128, 64, 3, 2, 2, 16>},
+      {"gemm_bf16_128x128x64_r2w4_m16", TILEC_FAMILY_GEMM, TILEC_BF16, 128, 128, 64, 4, 0, 2,
+       launch_gemm_bf16<128, 128, 64, 2, 2, 2, 16>},
+      // operands of any alignment, read in place (gemm_bf16_any.hip; unroll =
+      // register sets)
+      {"gemm_bf16_64x64x64_any", TILEC_FAMILY_GEMM, TILEC_BF16, 64, 64, 64, 4, 0, 4,
+       launch_any_or_generic<64, 64, 2, 2, 4, 2>},
+      {"gemm_bf16_128x64x64_any", TILEC_FAMILY_GEMM, TILEC_BF16, 128, 64, 64, 4, 0, 2,
+       launch_any_or_generic<128, 64, 2, 2, 2, 2>},
+      {"gemm_bf16_128x128x64_any", TILEC_FAMILY_GEMM, TILEC_BF16, 128, 128, 64, 8, 0, 4,
+       launch_any_or_generic<128, 128, 2, 4, 4, 1>},
+  };
+  *count = (int)(sizeof(t) / sizeof(t[0]));
+  return t;
+}
+
 }  // namespace tilec

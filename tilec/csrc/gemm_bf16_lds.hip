@@ -61,7 +61,12 @@ template <int BK, int MF>
 __device__ __forceinline__ int swz_a(int row) {
   return BK == 64 ? (row >> 1) & 7 : (row >> (MF == 16 ? 1 : 2)) & 3;
 }
-__device__ __forceinline__ int swz_b(int krow) { return (4 * (krow & 3)) ^ (2 * ((krow >> 3) & 1)); }
+// Rows of 64 elements (8 chunks, two rows per 256-byte bank line): the first
+// term takes bit 1 of the row only, bit 0 already being a bank half.
+template <int ROW_CHUNKS>
+__device__ __forceinline__ int swz_b(int krow) {
+  return (ROW_CHUNKS == 8 ? 4 * ((krow >> 1) & 1) : 4 * (krow & 3)) ^ (2 * ((krow >> 3) & 1));
+}
 
 // How one operand's tile (R rows of its outer dimension — M for x1, N for
 // x2 — by BK of K) sits in a stage buffer.
@@ -79,9 +84,11 @@ struct Stage {
   static constexpr int INSTR = CHUNKS / 64 / NW;  // DMA instructions per wave per step
   static constexpr int BYTES = R * BK * 2;
   static_assert(CHUNKS % (64 * NW) == 0, "DMA must divide evenly");
-  static_assert(KC || R % 128 == 0, "transposed-read swizzle needs rows of >= 16 chunks");
+  static_assert(KC || R == 64 || R % 128 == 0, "transposed-read swizzle covers rows of 8 or 16 n chunks");
   static_assert(!KC || BK == 32 || BK == 64, "row swizzle covers 4 or 8 chunks per row");
-  __device__ __forceinline__ static int swz(int row) { return KC ? swz_a<BK, MF>(row) : swz_b(row); }
+  __device__ __forceinline__ static int swz(int row) {
+    return KC ? swz_a<BK, MF>(row) : swz_b<ROW_CHUNKS>(row);
+  }
   // Stored row and logical chunk of physical chunk p.
   __device__ __forceinline__ static void chunk(int p, int& row, int& lc) {
     row = p / ROW_CHUNKS;
@@ -674,6 +681,14 @@ TILEC_LDS_VARIANT(256, 256, 64, 2, 2, 4, 16)
 TILEC_LDS_VARIANT(256, 256, 32, 4, 2, 4, 16)
 TILEC_LDS_VARIANT(256, 128, 64, 3, 4, 2, 16)
 TILEC_LDS_VARIANT(128, 128, 64, 4, 2, 4, 16)
+TILEC_LDS_VARIANT(64, 64, 64, 4, 2, 2, 32)
+TILEC_LDS_VARIANT(64, 64, 64, 4, 2, 2, 16)
+TILEC_LDS_VARIANT(128, 64, 64, 3, 2, 2, 32)
+TILEC_LDS_VARIANT(128, 64, 64, 3, 2, 2, 16)
+TILEC_LDS_VARIANT(64, 128, 64, 3, 2, 2, 32)
+TILEC_LDS_VARIANT(64, 128, 64, 3, 2, 2, 16)
+TILEC_LDS_VARIANT(128, 128, 64, 2, 2, 2, 32)
+TILEC_LDS_VARIANT(128, 128, 64, 2, 2, 2, 16)
 #undef TILEC_LDS_VARIANT
 
 }  // namespace tilec

@@ -23,6 +23,7 @@ const VariantDesc* gemm_bf16_variants(int* count);
 const VariantDesc* panel_variants(int* count);
 const VariantDesc* direct_variants(int* count);
 const VariantDesc* gemm_f32_x6_variants(int* count);
+const VariantDesc* gemm_bf16_small_variants(int* count);
 int64_t direct_effective_splits(int64_t K, int split_k);
 size_t skinny_counter_bytes(int dtype, int64_t M, int64_t N, int64_t K, int split_k);
 size_t skinny_workspace_bytes(int dtype, int64_t M, int64_t N, int64_t K, int split_k);
@@ -58,7 +59,7 @@ const std::vector<const VariantDesc*>& table() {
   static std::once_flag once;
   std::call_once(once, [] {
     for (auto fam : {skinny_variants, gemm_f32_variants, gemm_bf16_variants, panel_variants, direct_variants,
-                     gemm_f32_x6_variants}) {
+                     gemm_f32_x6_variants, gemm_bf16_small_variants}) {
       int n = 0;
       const VariantDesc* v = fam(&n);
       for (int i = 0; i < n; ++i) t.push_back(&v[i]);

@@ -107,6 +107,8 @@ def hip_configs(M, K, N, dtype="f32", layout=None):
             continue  # the panel kernel reads a row-major x2 (it runs the streaming kernel otherwise)
         if pad_variant(v) and not needs_pad(M, K, N, layout, code):
             continue  # aligned operands: the direct-to-LDS variants read them in place
+        if any_variant(v) and not needs_pad(M, K, N, layout, code):
+            continue  # aligned operands: the direct-to-LDS variants
         if planes_variant(v) and M <= 16:
             continue  # bound by reading x2: the streaming and direct kernels' work
         if v["family"] == _lib.FAMILY_SKINNY and rows_variant(v):
@@ -191,6 +193,12 @@ def pad_variant(v):
     direct-to-LDS tile kernel (csrc/gemm_f32.hip, launch_gemm_f32_pad;
     csrc/gemm_bf16.hip, launch_gemm_bf16_pad)."""
     return v["name"].endswith("_pad")
+
+
+def any_variant(v):
+    """Variants named *_any read bf16 operands of any element alignment in
+    place (csrc/gemm_bf16_any.hip)."""
+    return v["name"].endswith("_any")
 
 
 def planes_variant(v):

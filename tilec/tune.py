@@ -156,12 +156,13 @@ def falls_back(kernel, M, K, N, dtype, layout=0):
     multiples of 8 into that form and run the plain tile on the others.  The
     row-dot kernel (`x @ W.T`, M <= 4) shifts every 16-byte piece into place
     when K is not a whole number of 16-byte groups.  The pad variants exist
-    for the other shapes and never fall back."""
+    for the other shapes and never fall back, nor do the bf16 variants that
+    read any alignment (`*_any`)."""
     v = _variant_by_name()[kernel]
     if v["family"] == _lib.FAMILY_SKINNY and re.search(r"_t\d+_r\d+_", kernel) and not kernel.endswith(
             ("_c128", "_c256")):
         return not aligned(K, dtype)
-    if v["family"] != _lib.FAMILY_GEMM or kernel.endswith("_pad"):
+    if v["family"] != _lib.FAMILY_GEMM or kernel.endswith(("_pad", "_any")):
         return False
     if kernel.endswith("_kc") and M % 8 == 0 and N % 8 == 0 and K % 8 == 0:
         return False
@@ -385,17 +386,23 @@ def _bf16_stream(rng, count):
     return got
 
 
-def _mixed_stream(rng, count, dtype):
+def _mixed_stream(rng, count, dtype, large=False):
     """Products of one dtype in every layout: M in [17, 4096], K and N in
     [64, 8192] log-uniform, half of the K and N multiples of 64 as layer
     widths are — linear layers' forward and gradient products, where tile,
-    plane, split and alignment choices all meet."""
+    plane, split and alignment choices all meet.  `large`: each size in
+    [1024, 8192], three in four multiples of 64, up to 2^37 multiply-adds."""
     size = lambda lo, hi: round(2 ** rng.uniform(math.log2(lo), math.log2(hi)))
-    width = lambda v: v // 64 * 64 if v > 64 and rng.random() < 0.5 else v
+    width = lambda v: v // 64 * 64 if v > 64 and rng.random() < (0.75 if large else 0.5) else v
     got = set()
     while len(got) < count:
-        M, K, N = size(17, 4096), width(size(64, 8192)), width(size(64, 8192))
-        if 1 << 20 <= M * K * N <= 1 << 34 and max(M * K, K * N, M * N) <= 1 << 25:
+        if large:
+            M, K, N = (width(size(1024, 8192)) for _ in range(3))
+            ok = 1 << 32 <= M * K * N <= 1 << 37
+        else:
+            M, K, N = size(17, 4096), width(size(64, 8192)), width(size(64, 8192))
+            ok = 1 << 20 <= M * K * N <= 1 << 34 and max(M * K, K * N, M * N) <= 1 << 25
+        if ok:
             got.add((M, K, N, dtype, rng.choice((0, 1, 2, 2, 3))))
     return got
 
@@ -409,7 +416,8 @@ def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_nar
     (seed + 3), the row-tile kernel's, row-major `n_medium` medium
     outputs (seed + 4) and `n_narrow` narrow outputs over a long K
     (seed + 5), `n_bf16` bf16 tile GEMMs in random layouts (seed + 6), and
-    `n_mixed` products of each dtype in random layouts (seed + 7, + 8).
+    `n_mixed` products of each dtype in random layouts (seed + 7, + 8) and a
+    third as many large ones (seed + 9, + 10).
     None of UNSEEN_SHAPES is ever included."""
     rng = random.Random(seed)
     out = set(CONFIG_SHAPES)
@@ -441,6 +449,8 @@ def shapes(n=500, seed=0, n_layout=120, n_rows=40, n_tile=30, n_medium=80, n_nar
             _narrow_stream(random.Random(seed + 5), n_narrow)}
     more |= _bf16_stream(random.Random(seed + 6), n_bf16)
     more |= _mixed_stream(random.Random(seed + 7), n_mixed, "f32") | _mixed_stream(random.Random(seed + 8), n_mixed, "bf16")
+    more |= _mixed_stream(random.Random(seed + 9), n_mixed // 3, "f32", large=True)
+    more |= _mixed_stream(random.Random(seed + 10), n_mixed // 3, "bf16", large=True)
     unseen = {u + (0,) for u in UNSEEN_SHAPES}
     return sorted((out | lay | rows | tile | more) - unseen, key=lambda s: (s[0] * s[1] * s[2], s))
 
