@@ -22,6 +22,15 @@
 // (r = l / 16, q = l % 16) adds columns E q .. E q + E-1 of rows 4 r + u,
 // u < 4, and waves take interleaved blocks.  The 4 row slots of a wave meet
 // in shuffles, the waves in LDS.  Rows split across workgroups (grid y).
+// Rows that are not whole 16-byte groups (odd lengths and strides, offset
+// views) are read in 16-byte loads at the element's own alignment (kAny): read
+// element by element they were bound by the number of loads, 4 or 8 times as
+// many (on MI355X, rows of 4096 x 4097: fp32 31.0 -> 13.2 us, 5.1 TB/s, bf16
+// 24.5 -> 9.6; its columns 41.7 -> 21.4 and 39.0 -> 13.2).  Every load lies inside its row: a group past the end is moved back to
+// the row's last E elements, and the elements that belong to the group before
+// it are dropped (rows) or the lane's accumulators shifted (columns).  Rows
+// past the end load the last row again.  Only rows shorter than one group are
+// read element by element.
 // Split reductions combine deterministically: every workgroup publishes its
 // V partial sums, and the last to finish (completion counter) adds the S
 // partials in split order, spread over all its threads when V is small
@@ -101,6 +110,18 @@ __device__ bool split_tail(float& val, int V, int split, int S, int cell, int ce
   return true;
 }
 
+// How a 16-byte group is read: kAligned, one load of a group that never
+// straddles the end of a row; kAny, one load at any element alignment;
+// kElements, element by element.
+enum Access { kElements, kAny, kAligned };
+
+// 16 bytes at any alignment (a global load: buffer loads drop the address's
+// low two bits), non-temporal.
+__device__ __forceinline__ i32x4 load16_any(const char* base, uint32_t off) {
+  typedef i32x4 __attribute__((aligned(2))) i32x4_any;
+  return __builtin_nontemporal_load(reinterpret_cast<const i32x4_any*>(base + off));
+}
+
 // The 16-byte group of E elements at element c of the row `rs` is based at,
 // raw (bf16 as pairs, low half first): elements at or past n load zeros.
 // VEC: n and c are multiples of E, one 16-byte load; otherwise element by
@@ -140,7 +161,7 @@ __device__ __forceinline__ float elem(const i32x4& w, int e) {
 // Grid: x = groups of kWaves * 64 / lpr rows, y = column splits of `chunk`
 // columns (a multiple of 64 E).  U: 16-byte groups in flight per lane (16
 // for long rows, whose workgroup then reads 64 KiB of x at once).
-template <typename T, bool VEC, int U>
+template <typename T, Access ACC, int U>
 __global__ __launch_bounds__(kNT) void row_sum_kernel(const T* __restrict__ x, float* __restrict__ out, int R, int C,
                                                       int64_t ld, int lpr, int chunk, float* __restrict__ ws,
                                                       unsigned* __restrict__ counters) {
@@ -157,19 +178,57 @@ __global__ __launch_bounds__(kNT) void row_sum_kernel(const T* __restrict__ x, f
   const int cbeg = split * chunk;
   const int n = r < R ? max(0, min(C, cbeg + chunk) - cbeg) : 0;  // this split's columns of the row
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  // One resource per wave, at its first row (buffer resources are
-  // wave-uniform); a lane's row is a byte offset from it.
-  const BufRsrc rs = make_rsrc(x + (int64_t)(blockIdx.x * rpg + wave * rpw) * ld + cbeg);
-  const uint32_t row_off = (uint32_t)(lane / lpr) * (uint32_t)ld * (uint32_t)sizeof(T);
+  // One base per wave, at its first row (buffer resources are wave-uniform);
+  // a lane's row is a byte offset from it.
   const int step = E * lpr;
-  for (int c0 = E * sub; c0 < n; c0 += U * step) {
-    i32x4 w[U];
+  if constexpr (ACC == kAny) {
+    // Rows past R read row R - 1 (their sums are not stored), so the number
+    // of columns is the same for all lanes.  Offsets start `back` elements
+    // before the split's first column: its last group may begin there.
+    const int row0 = min((int)blockIdx.x * rpg + wave * rpw, R - 1);
+    const int cols = min(C, cbeg + chunk) - cbeg;
+    const int back = min(cbeg, E);
+    const char* base = reinterpret_cast<const char*>(x + (int64_t)row0 * ld + cbeg - back);
+    const uint32_t row_off =
+        ((uint32_t)min(lane / lpr, R - 1 - row0) * (uint32_t)ld + (uint32_t)back) * (uint32_t)sizeof(T);
+    int b = 0;  // the workgroup's first column of U groups per lane
+    for (; b + U * step <= cols; b += U * step) {
+      i32x4 w[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) w[u] = load_group<T, VEC>(rs, row_off, c0 + u * step, n);
+      for (int u = 0; u < U; ++u)
+        w[u] = load16_any(base, row_off + (uint32_t)(b + u * step + E * sub) * (uint32_t)sizeof(T));
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[e & 3] += elem<T>(w[u], e);
+        for (int e = 0; e < E; ++e) acc[e & 3] += elem<T>(w[u], e);
+    }
+    if (b < cols) {
+      i32x4 w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        w[u] = i32x4{0, 0, 0, 0};
+        if (b + u * step < cols)
+          w[u] = load16_any(base, row_off + (uint32_t)(min(b + u * step + E * sub, cols - E) * (int)sizeof(T)));
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int drop = b + u * step + E * sub - (cols - E);  // elements of the moved group that are others'
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[e & 3] += e >= drop ? elem<T>(w[u], e) : 0.f;
+      }
+    }
+  } else {
+    const BufRsrc rs = make_rsrc(x + (int64_t)(blockIdx.x * rpg + wave * rpw) * ld + cbeg);
+    const uint32_t row_off = (uint32_t)(lane / lpr) * (uint32_t)ld * (uint32_t)sizeof(T);
+    for (int c0 = E * sub; c0 < n; c0 += U * step) {
+      i32x4 w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = load_group<T, ACC == kAligned>(rs, row_off, c0 + u * step, n);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[e & 3] += elem<T>(w[u], e);
+    }
   }
   float s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   for (int o = lpr >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -189,7 +248,7 @@ __global__ __launch_bounds__(kNT) void row_sum_kernel(const T* __restrict__ x, f
 }
 
 // Grid: x = slabs of 16 E columns, y = row splits of kc rows (a multiple of 16).
-template <typename T, bool VEC>
+template <typename T, Access ACC>
 __global__ __launch_bounds__(kNT) void col_sum_kernel(const T* __restrict__ x, float* __restrict__ out, int R, int C,
                                                       int64_t ld, int kc, float* __restrict__ ws,
                                                       unsigned* __restrict__ counters) {
@@ -209,6 +268,10 @@ __global__ __launch_bounds__(kNT) void col_sum_kernel(const T* __restrict__ x, f
   // This lane's group: columns n0 + E q .. + E-1 of each row it adds; the
   // loader sees the row from n0 + E q, so `cn` columns of it are in x.
   const int cn = C - (n0 + E * q);
+  // kAny: the group's first column relative to n0 - back, moved back to lie
+  // inside the row.
+  const int back = min(n0, E);
+  const int col = min(E * q, C - E - n0) + back;
   float acc[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) acc[e] = 0.f;
@@ -217,6 +280,18 @@ __global__ __launch_bounds__(kNT) void col_sum_kernel(const T* __restrict__ x, f
 #pragma unroll
     for (int j = 0; j < UB; ++j) {
       const int b = b0 + j * kWaves;  // may be past the split: its rows load nothing
+      if constexpr (ACC == kAny) {
+        const int r0 = min(16 * b, nrows - 1);
+        const char* base = reinterpret_cast<const char*>(x + (int64_t)(rbeg + r0) * ld + n0 - back);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int row = 4 * r4 + u;
+          const uint32_t off = ((uint32_t)min(row, nrows - 1 - r0) * (uint32_t)ld + (uint32_t)col) * (uint32_t)sizeof(T);
+          w[j][u] = load16_any(base, off);
+          if (16 * b + row >= nrows) w[j][u] = i32x4{0, 0, 0, 0};
+        }
+        continue;
+      }
       // One resource per wave and block, at the block's first row and the
       // slab's first column (wave-uniform); a lane's row and columns are a
       // byte offset from it.  Rows past the split get n = 0.
@@ -226,7 +301,7 @@ __global__ __launch_bounds__(kNT) void col_sum_kernel(const T* __restrict__ x, f
         const int row = 4 * r4 + u;  // within the block
         const bool ok = 16 * b + row < nrows;
         const uint32_t off = ((uint32_t)row * (uint32_t)ld + (uint32_t)(E * q)) * (uint32_t)sizeof(T);
-        w[j][u] = load_group<T, VEC>(rs, off, 0, ok ? cn : 0);
+        w[j][u] = load_group<T, ACC == kAligned>(rs, off, 0, ok ? cn : 0);
       }
     }
 #pragma unroll
@@ -235,6 +310,12 @@ __global__ __launch_bounds__(kNT) void col_sum_kernel(const T* __restrict__ x, f
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int e = 0; e < E; ++e) acc[e] += elem<T>(w[j][u], e);
+  }
+  if constexpr (ACC == kAny) {  // a moved group's columns begin E - cn further up (past C: not stored)
+    for (int i = cn; i < E && i > 0; ++i) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[e] = e + 1 < E ? acc[e + 1] : 0.f;
+    }
   }
   // The 4 row slots of the wave (lanes q, q + 16, q + 32, q + 48), then the waves.
 #pragma unroll
@@ -306,8 +387,13 @@ ReduceGeom reduce_geom(int64_t R, int64_t C, int esz, int axis) {
     g.lpr = 0;
     g.cells = cdiv(std::max<int64_t>(C, 1), 16 * E);
     int64_t s = 1;
-    // Too few slabs: split rows, each split giving every wave at least 4 blocks.
-    if (g.cells < kFillWgs) s = std::max<int64_t>(1, std::min(cdiv(kFillWgs, g.cells), R / (16 * kWaves * 4)));
+    // Too few slabs: split rows, each split giving every wave at least the 2
+    // blocks it reads at a time, from 4 splits on (on MI355X, columns of 512 x
+    // 1000 fp32: 4.7 us, 5.6 in the 2 splits of 4 blocks a wave; of 1024 x
+    // 1000 bf16 4.8, 6.0 in 4).  Below that the combine costs more than it
+    // saves (256 x 1000 fp32: 3.9 us unsplit, 4.3 in 2 splits).
+    const int64_t most = R / (16 * kWaves * 2);
+    if (g.cells < kFillWgs && most >= 4) s = std::min(cdiv(kFillWgs, g.cells), most);
     g.span = std::max<int64_t>(16, cdiv(cdiv(R, s), 16) * 16);
     g.splits = std::max<int64_t>(1, cdiv(R, g.span));
   }
@@ -323,18 +409,18 @@ size_t reduce_counter_bytes(const ReduceGeom& g) {
 
 namespace {
 
-template <typename T, bool VEC>
+template <typename T, Access ACC>
 hipError_t launch_reduce_t(const void* x, float* out, int64_t R, int64_t C, int64_t ld, int axis, const ReduceGeom& g,
                            float* ws, unsigned* counters, hipStream_t stream) {
   const dim3 grid((unsigned)g.cells, (unsigned)g.splits);
   if (axis == 1 && g.lpr == 64)
-    hipLaunchKernelGGL((row_sum_kernel<T, VEC, 16>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out,
+    hipLaunchKernelGGL((row_sum_kernel<T, ACC, 16>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out,
                        (int)R, (int)C, ld, g.lpr, (int)g.span, ws, counters);
   else if (axis == 1)
-    hipLaunchKernelGGL((row_sum_kernel<T, VEC, 4>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out,
+    hipLaunchKernelGGL((row_sum_kernel<T, ACC, 4>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out,
                        (int)R, (int)C, ld, g.lpr, (int)g.span, ws, counters);
   else
-    hipLaunchKernelGGL((col_sum_kernel<T, VEC>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out, (int)R,
+    hipLaunchKernelGGL((col_sum_kernel<T, ACC>), grid, dim3(kNT), 0, stream, static_cast<const T*>(x), out, (int)R,
                        (int)C, ld, (int)g.span, ws, counters);
   return hipGetLastError();
 }
@@ -386,11 +472,14 @@ hipError_t launch_reduce(const void* x, float* out, int64_t R, int64_t C, int64_
     ws = nullptr;
     counters = nullptr;
   }
-  if (dtype == TILEC_BF16)
-    return vec ? launch_reduce_t<u16, true>(x, out, R, C, ld, axis, g, ws, counters, stream)
-               : launch_reduce_t<u16, false>(x, out, R, C, ld, axis, g, ws, counters, stream);
-  return vec ? launch_reduce_t<float, true>(x, out, R, C, ld, axis, g, ws, counters, stream)
-             : launch_reduce_t<float, false>(x, out, R, C, ld, axis, g, ws, counters, stream);
+  const Access acc = vec ? kAligned : R > 0 && C >= E ? kAny : kElements;
+  auto run = [&](auto zero) {
+    using T = decltype(zero);
+    return acc == kAligned ? launch_reduce_t<T, kAligned>(x, out, R, C, ld, axis, g, ws, counters, stream)
+           : acc == kAny   ? launch_reduce_t<T, kAny>(x, out, R, C, ld, axis, g, ws, counters, stream)
+                           : launch_reduce_t<T, kElements>(x, out, R, C, ld, axis, g, ws, counters, stream);
+  };
+  return dtype == TILEC_BF16 ? run(u16{}) : run(float{});
 }
 
 }  // namespace tilec
