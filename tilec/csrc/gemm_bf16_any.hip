@@ -238,6 +238,27 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_bf16_any_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  // The running sums move to a second set every FOLD K steps (256 k): a sum's
+  // rounding error grows as the root of the number of its additions, and the
+  // tiles with many K splits that this kernel takes over from kept theirs short.
+  constexpr int FOLD = 4;
+  f32x16 sum[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) sum[i][j] = acc[i][j];
+  auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          sum[i][j][r] += acc[i][j][r];
+          acc[i][j][r] = 0.f;
+        }
+  };
+
   const int half = lane >> 5;
   const int a_r = wm * WTM + (lane & 31), b_r = wn * WTN + (lane & 31);
   struct Frag {
@@ -312,6 +333,7 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_bf16_any_kernel(
         step(std::integral_constant<int, 2>{});
         step(std::integral_constant<int, 3>{});
       }
+      if ((s + PF) % FOLD == 0) fold();
     }
     if (s < nk) step(std::integral_constant<int, 0>{});
     if constexpr (PF > 2) {
@@ -319,6 +341,13 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_bf16_any_kernel(
       if (s + 2 < nk) step(std::integral_constant<int, 2>{});
     }
   }
+
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
 
   const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
   const int row_base = m0 + wm * WTM + 4 * half;

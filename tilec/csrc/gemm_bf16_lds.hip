@@ -309,6 +309,39 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_bf16_lds_kernel(
     for (int j = 0; j < P::TN; ++j)
 #pragma unroll
       for (int r = 0; r < P::ACC; ++r) acc[i][j][r] = 0.f;
+  // The four-wave tiles of up to 128 x 128 run few K splits where the tiles
+  // they take over from ran many, so their running sums move to a second set
+  // about every 256 k: a sum's rounding error grows as the root of the number
+  // of its additions.  Error against 64 bits at 128 x 4096 x 4096 (x @ W.T, 2
+  // splits): 2.7e-7 without, 1.1e-7 with; 1.4e-7 in 8 splits of 128 x 128.
+  // (A pass takes 11.4 and 12.3 us; 18.4 in 8 splits.)
+  constexpr bool FOLD = P::NT == 256 && BM <= 128 && BN <= 128;
+  constexpr int FOLD_RINGS = FOLD ? (256 + 64 * NBUF - 1) / (64 * NBUF) : 1;  // turns of the ring between folds
+  static_assert(!FOLD || BK == 64, "folds count 64-deep steps");
+  typename P::Acc sum[FOLD ? P::TM : 1][FOLD ? P::TN : 1];
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < P::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < P::TN; ++j) sum[i][j] = acc[i][j];
+  }
+  int rings = 0;
+  // After a turn of the ring.
+  auto fold = [&]() __attribute__((always_inline)) {
+    if constexpr (FOLD) {
+      if (++rings < FOLD_RINGS) return;
+      rings = 0;
+#pragma unroll
+      for (int i = 0; i < P::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < P::TN; ++j)
+#pragma unroll
+          for (int r = 0; r < P::ACC; ++r) {
+            sum[i][j][r] += acc[i][j][r];
+            acc[i][j][r] = 0.f;
+          }
+    }
+  };
 
   // Per-lane fragment addressing (bytes within an operand's stage area).
   // A fragment is 8 consecutive k of one of the wave's MF rows (MFMA operand
@@ -464,6 +497,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_bf16_lds_kernel(
     step(std::integral_constant<int, 1>{}, kt + 1);
     if constexpr (NBUF > 2) step(std::integral_constant<int, 2>{}, kt + 2);
     if constexpr (NBUF > 3) step(std::integral_constant<int, 3>{}, kt + 3);
+    fold();
   }
   // Remaining steps (fewer than NBUF): same slots in order.
   if (kt < nk) step(std::integral_constant<int, 0>{}, kt);
@@ -589,6 +623,7 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_bf16_lds_kernel(
       step16(std::integral_constant<int, 1>{}, kt + 1);
       if constexpr (NBUF > 2) step16(std::integral_constant<int, 2>{}, kt + 2);
       if constexpr (NBUF > 3) step16(std::integral_constant<int, 3>{}, kt + 3);
+      fold();
     }
     if (kt < nrun) step16(std::integral_constant<int, 0>{}, kt);
     if (kt + 1 < nrun) step16(std::integral_constant<int, 1>{}, kt + 1);
@@ -603,6 +638,14 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm_bf16_lds_kernel(
         for (int j = 0; j < P::TN; ++j) acc[x][j] = mfma_blk(fa[x], b[j], acc[x][j]);
     };
     mma_last(fb[0]);
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < P::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < P::TN; ++j)
+#pragma unroll
+        for (int r = 0; r < P::ACC; ++r) acc[i][j][r] += sum[i][j][r];
   }
   // Loads issued for steps past K still write (zeros) into LDS: let them
   // land before this workgroup can finish and release its LDS.
