@@ -808,6 +808,24 @@ def pick(M, K, N, dtype="f32", layout=0):
         return measured
     if model.keep is not None:
         cands = [c for c in cands if c[0] in model.keep] or cands
+    # A tile whose copies do not take these operands is out: the variants that
+    # read or pad any alignment cover them (over the timed shapes with such
+    # operands, the best of the rest is within 1.0001x of the best), and a
+    # prediction that misses the fallback costs up to 3x (1024 x 7287 x 3648).
+    by_name = _variant_by_name()
+    cands = [c for c in cands if by_name[c[0]]["family"] != _lib.FAMILY_GEMM
+             or not falls_back(c[0], M, K, N, dtype, layout)] or cands
+    # A 128x128 tile for every CU: the padded copies pay (the best `*_any` tile
+    # is best on 4 of 42 timed shapes, 0.76-0.87x of the best of the rest; on 323
+    # of 334 with fewer than 128 such tiles, 1.52x).
+    if cdiv(M, 128) * cdiv(N, 128) >= _cus():
+        cands = [c for c in cands if not c[0].endswith("_any")] or cands
+    # x @ W.T, both operands k-contiguous: the 64x64 plane kernel without LDS
+    # reads 32-byte pieces of 64 rows at a time, and its K splits are best on 4
+    # of the 77 timed shapes past 16 rows (by 3 % at most; 512 x 2048 x 1000,
+    # 26.0 us against 23.0 for the direct-to-LDS tile).
+    if layout == _lib.X2_COL_MAJOR:
+        cands = [c for c in cands if c[1] == 1 or not c[0].endswith("_d4_x6")] or cands
     cus = _cus()
     if model.n_features < len(features(M, K, N, cus, dtype, cands[0][0], cands[0][1], layout)):
         return None  # a model trained on fewer features than these: use the built-in rule
