@@ -9,7 +9,10 @@ a step is one `matrix_mul` call on resident, seeded U(-1,1) inputs; K steps
 are timed between HIP events on the stream the kernel runs on, after S ms of
 untimed calls (default 200: the GPU's clocks settle under sustained load)
 and W warmup steps.  Extra objects in the same line:
-  roofline     — the 4096^3 kernel against the fp32 MFMA peak (157.3 TFLOP/s)
+  roofline     — the 4096^3 kernel against the fp32 MFMA peak (157.3 TFLOP/s;
+                 the plane kernels run six bf16 products on the bf16 matrix
+                 cores instead and pass it: `frac_bf16_planes` is their share
+                 of that unit's peak / 6, 419 TFLOP/s)
   skinny       — the metric's "GB/s + %HBM roofline at M<=16" (config 1):
                  M in {1,4,16} fp32 and {1,16} bf16, K=N=4096, x2 rotated
                  over 512 MiB of copies (beyond the 256 MB Infinity Cache),
@@ -821,6 +824,7 @@ def main():
                    "M": 4096, "N": 4096, "K": 4096, "kernel": list(sq["config"])},
         "roofline": {"bound": "mfma", "achieved": round(sq["tflops"], 3), "peak": PEAK_FP32_MFMA,
                      "unit": "TFLOP/s", "frac": round(sq["tflops"] / PEAK_FP32_MFMA, 4),
+                     "frac_bf16_planes": round(6 * sq["tflops"] / PEAK_BF16_MFMA, 4),
                      "traffic": traffic_of(sq["config"][0], 4096, 4096, 4096)},
         "cpu_baseline": cpu,
         "device": {"name": props.name, "cus": props.multi_processor_count,
