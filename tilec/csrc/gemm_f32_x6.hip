@@ -9,9 +9,12 @@
 // large fp32 product on them is bound by that unit (137 GFLOP at 4096^3 take
 // 0.89 ms at its 157 TFLOP/s peak).  Here every fp32 value x is split exactly
 // into three bf16 planes,
-//   hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid),  x = hi + mid + lo
-// (8 significand bits each, round to nearest; both differences are exact),
-// and the product is the six plane products of relative size 2^-16 and up,
+//   y = 2^16 x, hi = bf16(y), mid = bf16(y - hi), lo = bf16(y - hi - mid),  y = hi + mid + lo
+// (8 significand bits each, round to nearest; both differences are exact; the
+// split and its six products are a published method: Henry, Tang and Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", ARITH 2019), and the product is the six
+// plane products of relative size 2^-16 and up,
 //   hi hi + (hi mid + mid hi) + (hi lo + mid mid + lo hi),
 // each exact in fp32 and accumulated in fp32: 6 x the MFMA work at 16 x the
 // rate.  The three dropped products are below 2^-24 of the term they belong
@@ -19,18 +22,23 @@
 // accumulator where the fp32 MFMA adds 2, so the result is closer to the
 // exact one than the fp32 MFMA's.
 //
-// Values the split does not hold: an infinity or NaN (or an overflow of hi,
-// above 3.39e38) makes its outputs non-finite; a row of x1 (column of x2) all
-// of whose values are below 2^-70 would lose low bits of its planes to
-// underflow, and one of each whose largest values multiply to less than 2^-96
-// low bits of the small products.  Each wave tests for these after its K loop
-// (its accumulators; the largest magnitude of its rows, gathered while they
-// are split) and then multiplies its part of the tile again on the fp32 MFMAs.
+// Range.  bf16 has the exponents of fp32 and 16 bits less, so the low planes of
+// a value under 2^-110 would fall below bf16's smallest subnormal, 2^-133.  The
+// factor 2^16 lifts every fp32 value, subnormals too, far enough (the least bit
+// of a subnormal, 2^-149, to 2^-133; the matrix cores keep bf16 and fp32
+// subnormals), and a product that is a normal fp32 number lifts the terms of
+// its plane products above 2^-142.  So the split is exact for every element on
+// its own, whatever else its row or column holds.  The sums are 2^32 times the
+// result and are multiplied by 2^-32 at the end.  What the factor takes is the
+// other end: a value of 2^112 (5e33) or a sum of 2^96 (8e28) overflows, as an
+// infinity or NaN would, into a sum that is not finite.  Each wave tests its
+// sums after the K loop and multiplies them again on the fp32 MFMAs if one is
+// such, which gives the fp32 kernels' results.
 //
 // Data movement.  A K step's tiles go global -> registers -> LDS: a thread
 // loads 8 consecutive k of one row ("chunk"; two 16-byte loads of a
 // k-contiguous operand, eight 4-byte loads along k of an r-contiguous one,
-// coalesced over lanes), splits them (5.5 VALU operations a value, beside the
+// coalesced over lanes), splits them (6.5 VALU operations a value, beside the
 // other waves' MFMAs) and stores three 16-byte chunks, which are the MFMA
 // operands as they are: LDS holds chunk (plane, kg, r) at
 // (plane KG + kg) R + (r ^ swz(kg)), so reads of 32 consecutive rows and the
@@ -61,13 +69,16 @@ namespace {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// 8 fp32 values -> three planes of 8 bf16 (hi, mid, lo), rounded to nearest.
+constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
+
+// 8 fp32 values -> three planes of 8 bf16 (hi, mid, lo) of kScale times them,
+// rounded to nearest.
 // (Splitting with integer adds and permutes, or with dot products by (-1, 0)
 // for the differences, measured level and 5 % slower.)
 __device__ __forceinline__ void split3(const float (&x)[8], u32x4 (&p)[3]) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float a = x[2 * j], b = x[2 * j + 1];
+    float a = kScale * x[2 * j], b = kScale * x[2 * j + 1];
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       uint32_t w = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)a, (__bf16)b});
@@ -120,18 +131,6 @@ __device__ __forceinline__ f32x4 load_f32x4_s(BufRsrc r, uint32_t voff, uint32_t
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
 
-constexpr float kTinyRow = 0x1p-70f, kTinyProduct = 0x1p-96f;
-
-// Least of the nonzero maxima of `rows` rows (all lanes of the wave get it).
-__device__ __forceinline__ void least_row(const uint32_t* rowmax, int rows, int lane, float& m) {
-  for (int i = lane; i < rows; i += 64) {
-    const float v = __uint_as_float(rowmax[i]);
-    m = v > 0.f ? fminf(m, v) : m;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fminf(m, __shfl_xor(m, o));
-}
-
 template <int BM, int BN, int BK, int WM, int WN, bool CA, bool CB>
 struct Gemm6 {
   static constexpr int NT = WM * WN * 64;
@@ -141,7 +140,7 @@ struct Gemm6 {
   using OB = Op6<BN, BK, NT, CB>;
   static constexpr int STAGE = OA::BYTES + OB::BYTES;
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be whole 32x32 blocks");
-  static_assert(3 * STAGE + 4 * (BM + BN) + 16 <= 160 * 1024, "LDS is 160 KiB");
+  static_assert(3 * STAGE + 16 <= 160 * 1024, "LDS is 160 KiB");
 };
 
 // Scheduling of one row block: its NM MFMAs in order, the LDS reads of the
@@ -169,7 +168,6 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
   using OB = typename P::OB;
   constexpr int TM = P::TM, TN = P::TN;
   __shared__ int last_flag;
-  __shared__ uint32_t rowmax[BM + BN];
   __shared__ __align__(16) char lds[3 * P::STAGE];
 
   const int tid = threadIdx.x;
@@ -188,8 +186,6 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
   const int nk = max(0, kt1 - kt0);
   const bool tail = nk > 0 && kt1 * BK > K;
   const int whole = nk - (tail ? 1 : 0);
-
-  for (int i = tid; i < BM + BN; i += P::NT) rowmax[i] = 0u;
 
   uint32_t off_a[OA::Q], off_b[OB::Q];
 #pragma unroll
@@ -276,27 +272,19 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
     }
   };
 
-  // Largest magnitude of each of this thread's rows (operand A, then B).
-  float mx_a[OA::Q], mx_b[OB::Q];
-#pragma unroll
-  for (int q = 0; q < OA::Q; ++q) mx_a[q] = 0.f;
-#pragma unroll
-  for (int q = 0; q < OB::Q; ++q) mx_b[q] = 0.f;
-  auto put = [&](auto op, const float (&x)[8], float& mx, int q, char* area) __attribute__((always_inline)) {
+  auto put = [&](auto op, const float (&x)[8], int q, char* area) __attribute__((always_inline)) {
     using O = decltype(op);
     int r, kg;
     O::coord(tid, q, r, kg);
     u32x4 p[3];
     split3(x, p);
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) mx = fmaxf(fmaxf(mx, fabsf(x[e])), fabsf(x[e + 1]));
     char* d = area + O::at(kg, r);
 #pragma unroll
     for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(d + 16 * O::PLANE * s) = p[s];
   };
   auto store = [&](int p, int c, char* st) __attribute__((always_inline)) {
-    if (c < OA::Q) put(OA{}, xa[p][c], mx_a[c], c, st);
-    else put(OB{}, xb[p][c - OA::Q], mx_b[c - OA::Q], c - OA::Q, st + OA::BYTES);
+    if (c < OA::Q) put(OA{}, xa[p][c], c, st);
+    else put(OB{}, xb[p][c - OA::Q], c - OA::Q, st + OA::BYTES);
   };
 
   f32x16 acc[TM][TN], low[LOW ? TM : 1][TN];
@@ -327,7 +315,7 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
   // The products of row block i, small ones first.  LOW: the five small ones
   // go to sums of their own, which meet the running sum after the K loop, so
   // that it is rounded once per 16 k and not six times.
-  auto block = [&](int i, const Planes& a, const Planes (&b)[TN]) __attribute__((always_inline)) {
+  auto row_block = [&](int i, const Planes& a, const Planes (&b)[TN]) __attribute__((always_inline)) {
     constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
     for (int q = 0; q < 6; ++q)
@@ -410,7 +398,7 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
               b[bs ^ 1][j] = read(OB{}, lds + (last_k ? nxt : cur) + OA::BYTES, b_r + 32 * j, last_k ? 0 : ks + 1);
           }
           chunks((I0 + 2) % PF, ks * TM + i, lds + nn);
-          block(i, a[as], b[bs]);
+          row_block(i, a[as], b[bs]);
           sched_block<6 * TN>();
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -446,30 +434,17 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
     }
   }
 
-  // Values the planes do not hold (see above): the tests, per wave.
-#pragma unroll
-  for (int q = 0; q < OA::Q; ++q) {
-    int r, kg;
-    OA::coord(tid, q, r, kg);
-    atomicMax(&rowmax[r], __float_as_uint(mx_a[q]));
-  }
-#pragma unroll
-  for (int q = 0; q < OB::Q; ++q) {
-    int r, kg;
-    OB::coord(tid, q, r, kg);
-    atomicMax(&rowmax[BM + r], __float_as_uint(mx_b[q]));
-  }
-  __syncthreads();
-  float least[2] = {__builtin_inff(), __builtin_inff()};
-  least_row(rowmax + wm * P::WTM, P::WTM, lane, least[0]);
-  least_row(rowmax + BM + wn * P::WTN, P::WTN, lane, least[1]);
-  bool redo = least[0] < kTinyRow || least[1] < kTinyRow || least[0] * least[1] < kTinyProduct;
+  // Sums that are not finite (see above): the wave's again.
+  bool redo = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) redo |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+      for (int r = 0; r < 16; ++r) {
+        redo |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+        acc[i][j][r] *= kUnscale;
+      }
   if (__ballot(redo) != 0) {
     clear(acc);
     const int k_end = min(K, kt1 * BK);
@@ -544,9 +519,8 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
   constexpr int T = 64, NT = 64 * W;
   constexpr int RS = T + 4;              // row stride of a wave's sums in LDS
   constexpr int ITEMS = T * T / 4 / NT;  // float4 results per thread
-  static_assert(T * T % (4 * NT) == 0 && W * T * RS * 4 + 8 * T + 64 <= 160 * 1024, "results divide, LDS fits");
+  static_assert(T * T % (4 * NT) == 0 && W * T * RS * 4 + 64 <= 160 * 1024, "results divide, LDS fits");
   __shared__ __align__(16) float sums[W * T * RS];
-  __shared__ uint32_t rowmax[2 * T];
   __shared__ int flag, last_flag;
 
   const int tid = threadIdx.x;
@@ -566,7 +540,6 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
   const bool tail = mine > 0 && kt1 * 16 > K && (kt1 - 1 - kt0) % W == wave;
   const int whole = mine - (tail ? 1 : 0);
 
-  for (int i = tid; i < 2 * T; i += NT) rowmax[i] = 0u;
   if (tid == 0) flag = 0;
   __syncthreads();
 
@@ -623,6 +596,20 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
     }
   };
 
+  // This wave's first step into set 0.
+  auto first_step = [&]() __attribute__((always_inline)) {
+    if (!tail) return load_step(0);
+    const int k0 = (kt1 - 1) * 16;
+    const BufRsrc sa = make_rsrc_uniform(base_a(kt1 - 1), 0x7FFFFFFFu);
+    const BufRsrc sb = make_rsrc_uniform(base_b(kt1 - 1), 0x7FFFFFFFu);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        x[0][c][e] = load_f32_s(c < 2 ? sa : sb, k0 + 8 * half + e < K ? off[c] : kOob,
+                                (c < 2 ? !CA : CB) ? 4u * e : c < 2 ? k_a[e] : k_b[e]);
+  };
+
   f32x16 acc[2][2];
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -633,7 +620,6 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   };
   clear();
-  float mx[4] = {0.f, 0.f, 0.f, 0.f};
   struct Planes {
     bf16x8 p[3];
   };
@@ -643,8 +629,6 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
     for (int c = 0; c < 4; ++c) {
       u32x4 q[3];
       split3(x[p][c], q);
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) mx[c] = fmaxf(fmaxf(mx[c], fabsf(x[p][c][e])), fabsf(x[p][c][e + 1]));
 #pragma unroll
       for (int s = 0; s < 3; ++s) d[c].p[s] = __builtin_bit_cast(bf16x8, q[s]);
     }
@@ -663,19 +647,7 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
   if (mine > 0) {
     // Step s multiplies f[s & 1] while step s + 1 is split into the other set
     // and the registers it came from are loaded for step s + 3.
-    if (tail) {
-      const int k0 = (kt1 - 1) * 16;
-      const BufRsrc sa = make_rsrc_uniform(base_a(kt1 - 1), 0x7FFFFFFFu);
-      const BufRsrc sb = make_rsrc_uniform(base_b(kt1 - 1), 0x7FFFFFFFu);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          x[0][c][e] = load_f32_s(c < 2 ? sa : sb, k0 + 8 * half + e < K ? off[c] : kOob,
-                                  (c < 2 ? !CA : CB) ? 4u * e : c < 2 ? k_a[e] : k_b[e]);
-    } else {
-      load_step(0);
-    }
+    first_step();
     load_step(1);
     split_all(0, f[0]);
     load_step(0);
@@ -697,23 +669,20 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
     if (s < mine) multiply(f[0]);
   }
 
-  // Values the planes do not hold: the staged kernel's tests, for the whole
-  // workgroup.
-#pragma unroll
-  for (int c = 0; c < 4; ++c) atomicMax(&rowmax[32 * c + l32], __float_as_uint(mx[c]));
-  bool bad = false;
+  // Sums that are not finite: the whole workgroup's again on the fp32 MFMAs.
+  bool redo = false;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
-  if (bad) flag = 1;
+      for (int r = 0; r < 16; ++r) {
+        redo |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+        acc[i][j][r] *= kUnscale;
+      }
+  if (redo) flag = 1;
   __syncthreads();
-  float least[2] = {__builtin_inff(), __builtin_inff()};
-  least_row(rowmax, T, lane, least[0]);
-  least_row(rowmax + T, T, lane, least[1]);
-  if (flag || least[0] < kTinyRow || least[1] < kTinyRow || least[0] * least[1] < kTinyProduct) {
+  if (flag) {
     clear();
 #pragma unroll 1
     for (int st = kt0 + wave; st < kt1; st += W) {
