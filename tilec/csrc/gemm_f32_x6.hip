@@ -32,8 +32,12 @@
 // result and are multiplied by 2^-32 at the end.  What the factor takes is the
 // other end: a value of 2^112 (5e33) or a sum of 2^96 (8e28) overflows, as an
 // infinity or NaN would, into a sum that is not finite.  Each wave tests its
-// sums after the K loop and multiplies them again on the fp32 MFMAs if one is
-// such, which gives the fp32 kernels' results.
+// sums after the K loop and multiplies the row blocks that hold such a one
+// again on the fp32 MFMAs, which gives them the fp32 kernels' results.  On
+// MI355X, 4096^3 in 256 x 256 tiles: 0.57 ms; one infinity in x1 0.71 ms
+// (every column tile redoes one row block); every sum NaN or above 2^96 1.45
+// to 1.54 ms.  The fp32 MFMA kernel takes 0.91 ms whatever the data.  (Without loads in
+// flight, and the wave's whole part at a time: 2.05 and 2.77 ms.)
 //
 // Data movement.  A K step's tiles go global -> registers -> LDS: a thread
 // loads 8 consecutive k of one row ("chunk"; two 16-byte loads of a
@@ -142,6 +146,79 @@ struct Gemm6 {
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be whole 32x32 blocks");
   static_assert(3 * STAGE + 16 <= 160 * 1024, "LDS is 160 KiB");
 };
+
+// c = TN 32 x 32 blocks of products over `len` k on the fp32 MFMAs, operands
+// straight from memory.  `a` and `b`: the tile's first row and column at the
+// first k; this lane's row and columns are byte offsets from there (kOob past
+// the end) of k = 4 half.  Eight k a step, half h of the wave takes
+// 4 h .. 4 h + 3; SETS steps of loads in flight.  KA, KB: k contiguous.
+template <int TN, bool KA, bool KB>
+__device__ __forceinline__ void fp32_block(f32x16 (&c)[TN], const float* a, const float* b, int64_t lda, int64_t ldb,
+                                           uint32_t off_a, const uint32_t (&off_b)[TN], int len, int half) {
+  constexpr int SETS = 4;
+  float xa[SETS][4], xb[SETS][TN][4];
+  uint32_t k_a[4], k_b[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    k_a[e] = KA ? 4u * e : to_scalar(4u * e * (uint32_t)lda);
+    k_b[e] = KB ? 4u * e : to_scalar(4u * e * (uint32_t)ldb);
+  }
+  auto four = [](auto kc, float (&x)[4], const BufRsrc& rs, uint32_t off, const uint32_t (&k)[4])
+      __attribute__((always_inline)) {
+    if constexpr (decltype(kc)::value) {
+      const f32x4 v = load_f32x4_s(rs, off, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = v[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = load_f32_s(rs, off, k[e]);
+    }
+  };
+  auto mma = [&](const float (&x)[4], const float (&y)[TN][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) c[j] = mfma32x32x2(x[e], y[j][e], c[j]);
+  };
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c[j][r] = 0.f;
+  const int64_t a_step = KA ? 8 : 8 * lda, b_step = KB ? 8 : 8 * ldb;
+  int left = len;  // k not loaded yet; loads past the last whole step return zeros
+  auto load = [&](int p) __attribute__((always_inline)) {
+    const uint32_t recs = left >= 8 ? 0x7FFFFFFFu : 0u;
+    const BufRsrc ra = make_rsrc_uniform(a, recs), rb = make_rsrc_uniform(b, recs);
+    four(std::bool_constant<KA>{}, xa[p], ra, off_a, k_a);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) four(std::bool_constant<KB>{}, xb[p][j], rb, off_b[j], k_b);
+    if (left >= 8) {
+      a += a_step;
+      b += b_step;
+      left -= 8;
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < SETS; ++p) load(p);
+#pragma unroll 1
+  for (int s = 0; s < len / 8; s += SETS)
+#pragma unroll
+    for (int p = 0; p < SETS; ++p) {
+      mma(xa[p], xb[p]);
+      load(p);
+    }
+  if (left > 0) {
+    const BufRsrc ra = make_rsrc_uniform(a, 0x7FFFFFFFu), rb = make_rsrc_uniform(b, 0x7FFFFFFFu);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = 4 * half + e < left;
+      xa[0][e] = load_f32_s(ra, in ? off_a : kOob, k_a[e]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) xb[0][j][e] = load_f32_s(rb, in ? off_b[j] : kOob, k_b[e]);
+    }
+    mma(xa[0], xb[0]);
+  }
+}
 
 // Scheduling of one row block: its NM MFMAs in order, the LDS reads of the
 // next operands behind the first ones, and behind every MFMA a few of the
@@ -434,39 +511,30 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
     }
   }
 
-  // Sums that are not finite (see above): the wave's again.
-  bool redo = false;
+  // Sums that are not finite (see above): their row blocks again.
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i) {
+    bool bad = false;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        redo |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+        bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
         acc[i][j][r] *= kUnscale;
       }
-  if (__ballot(redo) != 0) {
-    clear(acc);
-    const int k_end = min(K, kt1 * BK);
-#pragma unroll 1
-    for (int k = kt0 * BK; k < k_end; k += 2) {
-      const int kk = k + half;
-      float a[TM], b[TN];
+    if (__ballot(bad) == 0) continue;
+    const int ra = a_r + 32 * i;
+    const uint32_t fa =
+        m0 + ra < M ? 4u * (CA ? 4u * half * (uint32_t)lda + ra : (uint32_t)ra * (uint32_t)lda + 4u * half) : kOob;
+    uint32_t fb[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int r = m0 + a_r + 32 * i;
-        a[i] = r < M && kk < k_end ? A[CA ? (int64_t)kk * lda + r : (int64_t)r * lda + kk] : 0.f;
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int r = n0 + b_r + 32 * j;
-        b[j] = r < N && kk < k_end ? B[CB ? (int64_t)r * ldb + kk : (int64_t)kk * ldb + r] : 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32x32x2(a[i], b[j], acc[i][j]);
+    for (int j = 0; j < TN; ++j) {
+      const int rb = b_r + 32 * j;
+      fb[j] = n0 + rb < N ? 4u * (!CB ? 4u * half * (uint32_t)ldb + rb : (uint32_t)rb * (uint32_t)ldb + 4u * half) : kOob;
     }
+    fp32_block<TN, !CA, CB>(acc[i], !CA ? A + (int64_t)m0 * lda + (int64_t)kt0 * BK : A + (int64_t)kt0 * BK * lda + m0,
+                            CB ? B + (int64_t)n0 * ldb + (int64_t)kt0 * BK : B + (int64_t)kt0 * BK * ldb + n0, lda, ldb,
+                            fa, fb, min(K, kt1 * BK) - kt0 * BK, half);
   }
 
   const bool interior = (m0 + BM <= M) && (n0 + BN <= N);
@@ -669,7 +737,9 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
     if (s < mine) multiply(f[0]);
   }
 
-  // Sums that are not finite: the whole workgroup's again on the fp32 MFMAs.
+  // Sums that are not finite: the whole workgroup's again on the fp32 MFMAs,
+  // from the same loads (operand e of a chunk is k = e in one half of the wave
+  // and 8 + e in the other).
   bool redo = false;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -684,24 +754,29 @@ __global__ __launch_bounds__(W * 64, 2) void gemm_f32_x6_direct_kernel(
   __syncthreads();
   if (flag) {
     clear();
+    if (mine > 0) {
+      auto multiply32 = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x2(x[p][i][e], x[p][2 + j][e], acc[i][j]);
+      };
+      a_next = base_a(kt0 + wave);
+      b_next = base_b(kt0 + wave);
+      w = 0;
+      first_step();
+      load_step(1);
+      int s = 0;
 #pragma unroll 1
-    for (int st = kt0 + wave; st < kt1; st += W) {
-      const int k_end = min(K, 16 * st + 16);
-#pragma unroll 1
-      for (int k = 16 * st; k < k_end; k += 2) {
-        const int kk = k + half;
-        float a[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int r = m0 + 32 * i + l32, n = n0 + 32 * i + l32;
-          a[i] = r < M && kk < k_end ? A[CA ? (int64_t)kk * lda + r : (int64_t)r * lda + kk] : 0.f;
-          b[i] = n < N && kk < k_end ? B[CB ? (int64_t)n * ldb + kk : (int64_t)kk * ldb + n] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x2(a[i], b[j], acc[i][j]);
+      for (; s + 2 <= mine; s += 2) {
+        multiply32(0);
+        load_step(0);
+        multiply32(1);
+        load_step(1);
       }
+      if (s < mine) multiply32(0);
     }
   }
 
