@@ -190,16 +190,16 @@ int auto_variant(int64_t M, int64_t N, int64_t K, int dtype, int64_t ldx1, int64
       if (t64 >= cus && t64 <= 2 * (int64_t)cus) return find("gemm_f32_64x64x32_w2x2_lds");
       return find("direct_f32_32x64_w4_db");
     }
-    // Enough tiles to give every CU one: the plane kernels, unsplit (no
-    // scratch).  On MI355X, 4096^3: 0.59 ms in 256x256 tiles against 0.91 ms
-    // on the fp32 MFMAs; 2048^3, 256 tiles of 128x128: 116 against 126 us.
-    static const char* order[] = {"gemm_f32_256x256x16_x6", "gemm_f32_128x128x16_x6", "gemm_f32_128x64x16_w2x2"};
-    for (const char* nm : order) {
-      const int v = find(nm);
-      const VariantDesc* d = table()[v];
-      if (cdiv(M, d->bm) * cdiv(N, d->bn) >= cus) return v;
-    }
-    return find("gemm_f32_64x64x16_w2x2");
+    // A 128x128 tile for every CU (fewer were dealt with above, as 64x64 tiles
+    // are at most four times as many).  One or two products an output: the
+    // fp32 MFMAs, which round a single product correctly, where the planes'
+    // dropped terms add 0.9 of a rounding's error; and no slower on MI355X
+    // (4096 x 1 x 4096 17.0 us, 18.3 in plane tiles; 2048^2 7.9 and 9.7).
+    if (K <= 2) return find("gemm_f32_128x64x16_w2x2");
+    // The plane kernels, unsplit (no scratch): 4096^3 0.57 ms in 256x256 tiles
+    // against 0.91 ms on the fp32 MFMAs; 2048^3, 256 tiles of 128x128, 107
+    // against 126 us.
+    return find(cdiv(M, 256) * cdiv(N, 256) >= cus ? "gemm_f32_256x256x16_x6" : "gemm_f32_128x128x16_x6");
   }
   // bf16: the streaming kernel for M <= 16 (it runs fp32 MFMAs on widened
   // inputs, so more rows are better served by the bf16 tile GEMMs).
