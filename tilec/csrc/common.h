@@ -164,6 +164,23 @@ inline int device_xcds() {
   return x;
 }
 
+// Compute units of the current device (MI355X: 256; fewer in a partitioned
+// mode), read once per device; 256 if the query fails.
+inline int device_cus() {
+  constexpr int kMaxDev = 64;
+  static std::atomic<int> cache[kMaxDev];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev >= 0 && dev < kMaxDev) {
+    const int c = cache[dev].load(std::memory_order_relaxed);
+    if (c > 0) return c;
+  }
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+  if (dev >= 0 && dev < kMaxDev) cache[dev].store(cus, std::memory_order_relaxed);
+  return cus;
+}
+
 // Kernels with more than 64 KiB of dynamic LDS need their limit raised once
 // per device (the attribute belongs to the kernel on the current device).
 // `done` is the caller's per-kernel record of devices already set up

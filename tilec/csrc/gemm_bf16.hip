@@ -256,8 +256,8 @@ template <int BM, int BN, int WM, int WN>
 bool launch_unaligned(const MatmulArgs& a, hipError_t& e) {
   if (!any_takes(a)) return false;
   if (gemm_split_geom(a.K, 64, a.split_k).splits <= 1) {
-    e = cdiv(a.M, 128) * cdiv(a.N, 128) >= 256 ? launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a)
-                                               : launch_gemm_bf16_any<64, 64, 2, 2, 4, 2>(a);
+    e = cdiv(a.M, 128) * cdiv(a.N, 128) >= device_cus() ? launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a)
+                                                        : launch_gemm_bf16_any<64, 64, 2, 2, 4, 2>(a);
     return true;
   }
   if constexpr (BM == 128 && BN == 128 && WM == 2 && WN == 4) e = launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a);

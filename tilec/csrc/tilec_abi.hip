@@ -77,23 +77,6 @@ int find(const char* name) {
 
 constexpr int64_t kMaxDim = (int64_t(1) << 31) - 1024;  // kernels index rows/cols in int32
 
-// Compute units of the current device (MI355X: 256; fewer in a partitioned
-// mode), read once per device; 256 if the query fails.
-int device_cus() {
-  constexpr int kMaxDev = 64;
-  static std::atomic<int> cache[kMaxDev];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (dev >= 0 && dev < kMaxDev) {
-    const int c = cache[dev].load(std::memory_order_relaxed);
-    if (c > 0) return c;
-  }
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-  if (dev >= 0 && dev < kMaxDev) cache[dev].store(cus, std::memory_order_relaxed);
-  return cus;
-}
-
 // The skinny kernel addresses its operands within one block with 32-bit byte
 // offsets: row-major x2 over 16 rows (16 * ldx2 * 4 bytes < 2^31), x1 over 16
 // rows or (column-major) up to 32 columns of K (32 * ldx1 * 2 bytes), and
