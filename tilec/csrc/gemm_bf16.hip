@@ -252,9 +252,25 @@ bool any_takes(const MatmulArgs& a) {
 // 1024 with an x1 row stride of 1025, 43 against 17 us; 300 x 512 x 1024 with
 // one of 513, 44 against 6.8; 4096 x 1024 x 4096 with one of 1027, 174 against
 // 80).  A split keeps the variant's own tile, which its workspace is sized for.
+// One K step that is not nearly whole (K <= 56) stays on the generic kernel
+// where that is the faster: its 64 x 64 tile for x @ W.T (8 x 27 x 2049 4.4
+// against 4.8 us) and for row-major operands and more than two tiles a CU
+// (2049 x 17 x 1337 8.2 against 9.5), its 128 x 128 tile for an x @ W.T with
+// too few of them for every CU that has so many 64 x 64 ones (2049 x 27 x 1337
+// 8.9 against 10.0).
+template <int BM, int BN, int WM, int WN>
+bool generic_is_faster(const MatmulArgs& a) {
+  if (a.K > 56) return false;
+  const bool xwt = (a.layout & 3) == TILEC_X2_COL_MAJOR;
+  const bool many = cdiv(a.M, 64) * cdiv(a.N, 64) > 2 * device_cus();
+  if constexpr (BM == 64 && BN == 64) return xwt || (many && (a.layout & 3) == 0);
+  else if constexpr (BM == 128 && BN == 128) return xwt && many && cdiv(a.M, 128) * cdiv(a.N, 128) < device_cus();
+  else return false;
+}
+
 template <int BM, int BN, int WM, int WN>
 bool launch_unaligned(const MatmulArgs& a, hipError_t& e) {
-  if (!any_takes(a)) return false;
+  if (!any_takes(a) || generic_is_faster<BM, BN, WM, WN>(a)) return false;
   if (gemm_split_geom(a.K, 64, a.split_k).splits <= 1) {
     e = cdiv(a.M, 128) * cdiv(a.N, 128) >= device_cus() ? launch_gemm_bf16_any<128, 128, 2, 4, 4, 1>(a)
                                                         : launch_gemm_bf16_any<64, 64, 2, 2, 4, 2>(a);
