@@ -391,8 +391,11 @@ ReduceGeom reduce_geom(int64_t R, int64_t C, int esz, int axis) {
     // blocks it reads at a time, from 4 splits on (on MI355X, columns of 512 x
     // 1000 fp32: 4.7 us, 5.6 in the 2 splits of 4 blocks a wave; of 1024 x
     // 1000 bf16 4.8, 6.0 in 4).  Below that the combine costs more than it
-    // saves (256 x 1000 fp32: 3.9 us unsplit, 4.3 in 2 splits).
-    const int64_t most = R / (16 * kWaves * 2);
+    // saves (256 x 1000 fp32: 3.9 us unsplit, 4.3 in 2 splits).  Past 32 such
+    // splits 4 blocks a wave: the combine reads every split's partials alone
+    // (65536 x 8 bf16: 12.3 us in 256 splits, 20.1 in 512; 10000 x 8 5.7 in
+    // 39, 6.5 in 78).
+    const int64_t most = std::max<int64_t>(std::min<int64_t>(R / (16 * kWaves * 2), 32), R / (16 * kWaves * 4));
     if (g.cells < kFillWgs && most >= 4) s = std::min(cdiv(kFillWgs, g.cells), most);
     g.span = std::max<int64_t>(16, cdiv(cdiv(R, s), 16) * 16);
     g.splits = std::max<int64_t>(1, cdiv(R, g.span));
