@@ -109,17 +109,11 @@ def hip_configs(M, K, N, dtype="f32", layout=None):
             continue  # aligned operands: the direct-to-LDS variants read them in place
         if any_variant(v) and not needs_pad(M, K, N, layout, code):
             continue  # aligned operands: the direct-to-LDS variants
-        if v["family"] == _lib.FAMILY_GEMM and M <= 16 and N < 64:
-            continue  # a part of one tile: 4 x 6272 x 27 bf16, 12.1 us against the streaming kernel's 8.6
         if planes_variant(v) and M <= 16:
             continue  # bound by reading x2: the streaming and direct kernels' work
         if v["family"] == _lib.FAMILY_SKINNY and rows_variant(v):
             epl = 4 if code == _lib.F32 else 8  # elements per 16-byte load
             row_tile = v["name"].endswith(("_c128", "_c256"))  # the row-dot kernel takes any K
-            if N < 64 and K >= 4096 and K % epl:
-                # few waves, each shifting a whole row into place: 4 x 12697 x 18 bf16, 60 us, 8.8 on the
-                # streaming kernel's K splits (aligned, 1 x 5824 x 31: 3.2 us, 9.2 there)
-                continue
             if (K % epl == 0 or not row_tile) and (layout is None or layout == _lib.X2_COL_MAJOR):
                 out.append((v["name"], 1))  # neither kernel splits K
         elif v["family"] == _lib.FAMILY_DIRECT:
