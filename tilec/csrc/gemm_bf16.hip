@@ -252,15 +252,15 @@ bool any_takes(const MatmulArgs& a) {
 // 1024 with an x1 row stride of 1025, 43 against 17 us; 300 x 512 x 1024 with
 // one of 513, 44 against 6.8; 4096 x 1024 x 4096 with one of 1027, 174 against
 // 80).  A split keeps the variant's own tile, which its workspace is sized for.
-// One K step that is not nearly whole (K <= 56) stays on the generic kernel
+// One K step that is not nearly whole (K <= 60) stays on the generic kernel
 // where that is the faster: its 64 x 64 tile for x @ W.T (8 x 27 x 2049 4.4
-// against 4.8 us) and for row-major operands and more than two tiles a CU
+// against 4.8 us, 6 x 60 x 1069 4.0 against 4.6; 8 x 63 x 2049 4.5 against 4.2) and for row-major operands and more than two tiles a CU
 // (2049 x 17 x 1337 8.2 against 9.5), its 128 x 128 tile for an x @ W.T with
 // too few of them for every CU that has so many 64 x 64 ones (2049 x 27 x 1337
 // 8.9 against 10.0).
 template <int BM, int BN, int WM, int WN>
 bool generic_is_faster(const MatmulArgs& a) {
-  if (a.K > 56) return false;
+  if (a.K > 60) return false;
   const bool xwt = (a.layout & 3) == TILEC_X2_COL_MAJOR;
   const bool many = cdiv(a.M, 64) * cdiv(a.N, 64) > 2 * device_cus();
   if constexpr (BM == 64 && BN == 64) return xwt || (many && (a.layout & 3) == 0);

@@ -18,8 +18,9 @@
 // PF register sets (steps) ahead of the LDS store, which itself is two steps
 // ahead of the MFMAs (three LDS stages, one barrier a step; a step's first
 // operands are read before the barrier that ends the step before it).
-// LDS holds chunk (kg, r) (8 consecutive k of row r) at kg R + (r ^ kg): reads
-// of 32 consecutive rows and both kinds of store are free of bank conflicts.
+// LDS holds chunk (kg, r) (8 consecutive k of row r) at kg R + (r ^ kg), which
+// spreads 32 consecutive rows over all banks (300 x 2051 x 1001 row-major: 2 %
+// of the cycles in bank conflicts).
 //
 // Edges: rows past M or N are clamped to the last (their results are not
 // stored); a pair of columns past the end is moved down to the last pair (the
@@ -238,10 +239,15 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_bf16_any_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  // The running sums move to a second set every FOLD K steps (256 k): a sum's
-  // rounding error grows as the root of the number of its additions, and the
-  // tiles with many K splits that this kernel takes over from kept theirs short.
-  constexpr int FOLD = 4;
+  // The running sums move to a second set every 256 k, in the 64 x 64 tile every
+  // 128 up to 2048 k (beyond, the second set's additions count for more): a
+  // sum's rounding error grows as the root of the number of its additions, and
+  // the tiles and streaming kernels with many K splits that this kernel takes
+  // over from kept theirs short.  14 x 1538 x 1050 (x @ W.T, 4 splits): 9.3e-8
+  // with folds of 256 k, 8.5e-8 with 128 (7.5 us both), 9.0e-8 on the streaming
+  // kernel (11.5 us).  In the larger tiles folds of 128 k cost 4 to 5 % (300 x
+  // 2051 x 1001 in 128 x 64: 20.8 and 21.7 us).
+  const bool fine = BM == 64 && nk <= 32;
   f32x16 sum[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -329,11 +335,12 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_bf16_any_kernel(
     for (; s + PF <= nk; s += PF) {
       step(std::integral_constant<int, 0>{});
       step(std::integral_constant<int, 1>{});
+      if (fine) fold();
       if constexpr (PF > 2) {
         step(std::integral_constant<int, 2>{});
         step(std::integral_constant<int, 3>{});
       }
-      if ((s + PF) % FOLD == 0) fold();
+      if ((PF > 2 || !fine) && (s + PF) % 4 == 0) fold();
     }
     if (s < nk) step(std::integral_constant<int, 0>{});
     if constexpr (PF > 2) {

@@ -19,8 +19,9 @@
 // each exact in fp32 and accumulated in fp32: 6 x the MFMA work at 16 x the
 // rate.  The three dropped products are below 2^-24 of the term they belong
 // to, half an ulp of it, and the MFMA adds 16 products per rounding of the
-// accumulator where the fp32 MFMA adds 2, so the result is closer to the
-// exact one than the fp32 MFMA's.
+// accumulator where the fp32 MFMA adds 2, so from 3 products an output on the
+// result is closer to the exact one than the fp32 MFMA's (1 or 2 products:
+// 3.5e-8 and 2.6e-8, without and with LOW, against 2.5e-8 to 3.2e-8).
 //
 // Range.  bf16 has the exponents of fp32 and 16 bits less, so the low planes of
 // a value under 2^-110 would fall below bf16's smallest subnormal, 2^-133.  The
@@ -56,10 +57,12 @@
 // so the loop has no edge in K.
 //
 // Measured on MI355X against the fp32 MFMA kernels: 4096^3 565 against 914 us
-// (256 x 256, 8 waves; matrix cores 84 % busy at 1.75 GHz, the power limit;
-// relative error 1.0e-6 against 1.1e-6), 2048^3 104 against 126 us (128 x 128,
+// (256 x 256, 8 waves; matrix cores 76 % busy at 1.77 GHz, the power limit;
+// relative error 1.0e-6 against 1.1e-6), 2048^3 94 against 126 us (128 x 128,
 // 8 waves; error 2.7e-7 against 8.1e-7), 1000 x 4097 x 3001 143 against 204 us
 // (128 x 128, 4 waves, two workgroups a CU, K split 4; no padding copies).
+// Those 128-tiles keep the matrix cores 48 and 51 % busy, with 5 VALU
+// instructions an MFMA (2.4 in the 256-tile).
 // The 128-tiles keep the five small products in sums of their own (LOW),
 // which their registers allow; the 256-tile's do not.
 #include <type_traits>
@@ -563,12 +566,12 @@ __global__ __launch_bounds__(WM * WN * 64, WPE) void gemm_f32_x6_kernel(
 // of the workgroup's.  Every wave loads its own operands straight into
 // registers (chunks of 8 consecutive k, which split into MFMA operands as
 // they are), so the K loop has no barrier, no LDS traffic and no wait but for
-// its own loads; the waves' sums meet in LDS in wave order.  VALU issue bounds
-// a step: on MI355X 11 VALU operations an MFMA keep the SIMD's issue 80 % busy
-// at 56 % of the MFMA rate (4096^3).  1024^3: 17.5 us, against 20.5 on the
-// fp32 MFMAs (direct-to-LDS 64 x 64) and 22.5 for a staged 64 x 64 tile of the
+// its own loads; the waves' sums meet in LDS in wave order.  A step
+// issues 10 VALU instructions an MFMA.  On MI355X, 1024^3 back to back: 22 us
+// (the direct-to-LDS 64 x 64 tile on the fp32 MFMAs 23), error 2.4e-7 against
+// 5.7e-7; 512 x 1000 x 2048 20.2 us, 27.0 for a staged 64 x 64 x 32 tile of the
 // kernel above.  A ring of direct-to-LDS copies in front of the registers
-// measured no faster (19.5 us).
+// measured no faster.
 // ---------------------------------------------------------------------------
 template <int NM, int X = 0>
 __device__ __forceinline__ void sched_direct() {

@@ -1028,7 +1028,7 @@ def _offered(cands, M, K, N, dtype, layout):
     # So is the generic 64x64 bf16 tile, which runs the kernel of the `*_any`
     # tile for such operands, but for K steps too short for that one.
     by_name = _variant_by_name()
-    whole = dtype == "f32" or K <= 56 or (aligned(M if layout & _lib.X1_COL_MAJOR else K, dtype) and
+    whole = dtype == "f32" or K <= 60 or (aligned(M if layout & _lib.X1_COL_MAJOR else K, dtype) and
                                           aligned(K if layout & _lib.X2_COL_MAJOR else N, dtype))
     cands = [c for c in cands if by_name[c[0]]["family"] != _lib.FAMILY_GEMM
              or not (falls_back(c[0], M, K, N, dtype, layout) or
