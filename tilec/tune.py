@@ -1004,7 +1004,7 @@ def reference(M, K, N, dtype="f32", layout=0, table=True):
     if base is None or 0 in (M, K, N):
         return None
     from . import ext
-    cands = [c for c in ext.hip_configs(M, K, N, dtype, layout) if c[0] in base.keep]
+    cands = [c for c in ext.hip_configs(M, K, N, dtype, layout) if base.keep is None or c[0] in base.keep]
     if not cands:
         return None
     measured = base.best.get((M, K, N, dtype, layout)) if table else None
