@@ -1,5 +1,5 @@
-"""`tune.pick` leaves the reference model's choice only for a config whose sums
-are measured to be no less exact."""
+"""`tune.pick` leaves the more exact choice of the two reference models only for
+a config whose sums are measured to be no less exact."""
 
 import math
 import random
@@ -27,6 +27,13 @@ CASES = [
     ((1344, 4187, 2685, "bf16", 1), ("gemm_bf16_256x128x64_r3_m16_pad", 2)),
     ((128, 4096, 4096, "bf16", 2), None),
     ((1000, 4097, 3001, "f32", 0), None),
+    # more exact configs of the later kernels
+    ((4096, 16, 4096, "f32", 0), ("gemm_f32_256x256x16_x6", 1)),
+    ((382, 117, 2954, "f32", 2), ("gemm_f32_64x64x16_d4_x6", 1)),
+    ((606, 1732, 3584, "f32", 2), ("gemm_f32_128x128x16_x6", 4)),
+    ((128, 4822, 1792, "f32", 2), ("gemm_f32_128x128x32_w8_x6", 16)),
+    ((358, 6948, 4111, "bf16", 0), ("gemm_bf16_128x128x64_any", 4)),
+    ((640, 13184, 1245, "bf16", 1), ("gemm_bf16_128x128x64_any", 4)),
 ]
 
 
